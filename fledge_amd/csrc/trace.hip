@@ -38,7 +38,6 @@ FLG_D StackOf<RING> make_stack(uint2* ring, int stride, uint2* priv) {
 // scratch, which measured faster than the 4-5 waves of the unconstrained
 // allocation.
 constexpr int kTraceWaves = 8;
-constexpr uint32_t kCus = 256;  // of the chip
 
 template <bool COMPAT, int BS, int RING>
 __global__ __launch_bounds__(BS, kTraceWaves) void k_trace(TraceGeom g, const flg_ray* rays, flg_hit* hits,
@@ -316,9 +315,15 @@ __global__ __launch_bounds__(BS, kTraceWaves) void k_pt_bounce(TraceGeom g, PtSt
 
 // Bounces after the first, split in two launches (ray_fetch 2).  The
 // traversal kernel hands out the queue (its length is read on the device) in
-// chunks of kChunk rays, in queue order, through one counter per bounce: the
-// rays in flight at any moment then lie close together in the queue, which
-// follows the image, so they cross the same nodes and share the caches.
+// chunks of at most kChunk rays, in queue order: every wave starts with the
+// chunk of its own number and takes further ones through one counter per
+// bounce.  The rays in flight at any moment then lie close together in the
+// queue, which follows the image, so they cross the same nodes and share the
+// caches.  The grid is no larger than what the device holds at once: each wave
+// that found the queue empty through the counter cost about 4 ns there, one
+// after another, and with 64 blocks per CU that was most of a small mesh's time
+// (2,048 triangles, 1280 x 720 at 4 spp: 563 us with 32,768 waves and every
+// chunk from the counter, 205 us now).
 // Within a chunk a lane whose ray has ended takes the next entry whenever
 // enough of the wave's lanes are idle, so a wave does not idle behind its
 // longest traversal.  It only writes each ray's closest hit.  The shading
@@ -332,18 +337,19 @@ constexpr uint32_t kChunkMin = 8;
 // even share, at most `most`.  A short queue in chunks of 128 left most waves
 // without any and the others with two rays per lane, one after the other, each
 // a chain of dependent fetches: with shares of at least 8 rays, 0.93 M paths of
-// depth 4 on 0.5 M triangles take 1.50 ms against 1.68 ms (at least 16: 1.56,
-// 32: 1.59, 64: 1.61 ms).
+// depth 4 on 0.5 M triangles took 1.50 ms against 1.68 ms (at least 16: 1.56,
+// 32: 1.59, 64: 1.61 ms; every chunk from the counter then).
 FLG_D uint32_t queue_share(uint32_t n, uint32_t waves, uint32_t least, uint32_t most) {
   const uint32_t s = (n + waves - 1) / waves;
   return s < least ? least : s > most ? most : s;
 }
 
-// Takes the wave's next chunk [next, end) of a queue of n rays; false when
-// none is left.  Called by every lane of the wave together.
-FLG_D bool take_chunk(uint32_t* taken, uint32_t n, uint32_t chunk, uint32_t& next, uint32_t& end) {
+// Takes the wave's next chunk [next, end) of a queue of n rays beyond the first
+// `waves` ones; false when none is left.  Called by every lane of the wave
+// together.
+FLG_D bool take_chunk(uint32_t* taken, uint32_t n, uint32_t chunk, uint32_t waves, uint32_t& next, uint32_t& end) {
   uint32_t c = 0;
-  if ((threadIdx.x & 63) == 0) c = atomicAdd(taken, 1u);
+  if ((threadIdx.x & 63) == 0) c = waves + atomicAdd(taken, 1u);
   c = __builtin_amdgcn_readfirstlane(c);  // a scalar: the chunk bounds stay in SGPRs
   if (c >= (uint32_t)(((uint64_t)n + chunk - 1) / chunk)) return false;
   next = c * chunk;
@@ -351,7 +357,7 @@ FLG_D bool take_chunk(uint32_t* taken, uint32_t n, uint32_t chunk, uint32_t& nex
   return true;
 }
 
-constexpr int kSplitTraceWaves = 7;
+constexpr int kSplitTraceWaves = 7;  // per SIMD
 
 template <bool COMPAT, int BS, int RING>
 __global__ __launch_bounds__(BS, kSplitTraceWaves) void k_pt_trace(TraceGeom g, PtState s, int bounce) {
@@ -359,9 +365,12 @@ __global__ __launch_bounds__(BS, kSplitTraceWaves) void k_pt_trace(TraceGeom g, 
   const uint32_t n = s.count[bounce];
   const QRay* qin = s.q[bounce & 1];
   const int lane = threadIdx.x & 63;
-  const uint32_t chunk = queue_share(n, kCus * 4 * kSplitTraceWaves, kChunkMin, kChunk);
-  uint32_t next = 0, end = 0;  // the wave's current chunk; the same in every lane
-  bool more = true;            // chunks may be left
+  const uint32_t waves = gridDim.x * (BS / 64);
+  const uint32_t chunk = queue_share(n, waves, kChunkMin, kChunk);
+  // the wave's current chunk; the same in every lane
+  uint32_t next = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (BS / 64) + threadIdx.x / 64)) * chunk;
+  uint32_t end = next + chunk < n ? next + chunk : n;
+  bool more = (uint64_t)waves * chunk < n;  // chunks may be left beyond the waves' first ones
   uint2 priv[kStack];
   auto st = make_stack<RING>(ring + threadIdx.x, BS, priv);
   Counters c{0, 0};
@@ -374,7 +383,7 @@ __global__ __launch_bounds__(BS, kSplitTraceWaves) void k_pt_trace(TraceGeom g, 
   // chunk is left and all its lanes are idle; each traversal ends (a node is
   // visited at most once)
   while (true) {
-    if (next >= end && more) more = take_chunk(s.taken + bounce, n, chunk, next, end);
+    if (next >= end && more) more = take_chunk(s.taken + bounce, n, chunk, waves, next, end);
     const uint64_t idle = __ballot(r.node == kEnded);
     const bool all = __ballot(r.node != kEnded) == 0;
     if (all || (next < end && __popcll(idle) >= kRefillIdle)) {
@@ -501,7 +510,7 @@ constexpr int kPathWaves = 4;
 
 template <bool COMPAT, int BS, int RING>
 __global__ __launch_bounds__(BS, kPathWaves) void k_pt_paths(TraceGeom g, PtState s, HaltonTables tab,
-                                                 HaltonParams hp, int bounce0, int max_depth) {
+                                                 HaltonParams hp, int bounce0, int max_depth, uint32_t resident) {
   __shared__ uint2 ring[RING > 0 ? BS * RING : 1];
   const uint32_t n = s.count[bounce0];
   const QRay* qin = s.q[bounce0 & 1];
@@ -509,7 +518,7 @@ __global__ __launch_bounds__(BS, kPathWaves) void k_pt_paths(TraceGeom g, PtStat
   const uint32_t nwaves = gridDim.x * (BS / 64);
   const uint32_t wave = blockIdx.x * (BS / 64) + threadIdx.x / 64;
   uint32_t per = (uint32_t)(((uint64_t)n + nwaves - 1) / nwaves);
-  const uint32_t least = queue_share(n, kCus * 4 * kPathWaves, kSliceMin, kMinSlice);
+  const uint32_t least = queue_share(n, resident, kSliceMin, kMinSlice);
   per = per < least ? least : per;
   const uint64_t lo = (uint64_t)wave * per;
   const uint32_t end = (uint32_t)(lo + per < n ? lo + per : n);
@@ -587,9 +596,10 @@ constexpr int kRingDefault = 8;
 
 // Shapes of a call that names none on a context that was not tuned: what the
 // tuner picks on large frames.  Path tracer, the 2M-triangle frame
-// at 1920 x 1080: 7.7 ms against 14.1 ms with one fused launch per bounce, 256
+// at 1920 x 1080: 7.4 ms against 14.1 ms with one fused launch per bounce, 256
 // threads, 8 blocks per CU and private stacks; 0.93 M paths of depth 4 on 0.5 M
-// triangles: 1.52 against 1.54 ms.  Single rays: 500 against 525 us (1 M camera
+// triangles: 1.26 against 1.54 ms; 3.7 M paths of depth 8 on 2,048 triangles:
+// 0.75 against 0.83 ms.  Single rays: 500 against 525 us (1 M camera
 // rays on 65,536 triangles), 722 against 790 us (1 M unordered on 2 M).
 constexpr int kDefaultTraceBlock = 64, kDefaultStack = 2;
 constexpr int kDefaultPtBlock = 128, kDefaultPtBlocksPerCu = 64, kDefaultPtFetch = 4;
@@ -652,7 +662,9 @@ void launch_bounce_bs(int grid, int block, hipStream_t st, const TraceGeom& g, c
 }
 
 template <bool COMPAT, int RING>
-void launch_split_bs(int grid, int block, hipStream_t st, const TraceGeom& g, const PtState& s, int b) {
+void launch_split_bs(int cus, int blocks, int block, hipStream_t st, const TraceGeom& g, const PtState& s, int b) {
+  // no more waves than the device holds at once: the others would only find the queue empty
+  const int grid = std::min(blocks, cus * 4 * kSplitTraceWaves * 64 / block);
   switch (block) {
     case 64: k_pt_trace<COMPAT, 64, RING><<<grid, 64, 0, st>>>(g, s, b); break;
     case 128: k_pt_trace<COMPAT, 128, RING><<<grid, 128, 0, st>>>(g, s, b); break;
@@ -664,15 +676,16 @@ void launch_split_bs(int grid, int block, hipStream_t st, const TraceGeom& g, co
 }
 
 template <bool COMPAT, int RING>
-void launch_paths_bs(int grid, int block, hipStream_t st, const TraceGeom& g, const PtState& s,
+void launch_paths_bs(int cus, int grid, int block, hipStream_t st, const TraceGeom& g, const PtState& s,
                      const HaltonTables& tab, const HaltonParams& hp, int b, int D) {
+  const uint32_t waves = (uint32_t)cus * 4 * kPathWaves;  // that the device holds at once
   switch (block) {
-    case 64: k_pt_paths<COMPAT, 64, RING><<<grid, 64, 0, st>>>(g, s, tab, hp, b, D); break;
-    case 128: k_pt_paths<COMPAT, 128, RING><<<grid, 128, 0, st>>>(g, s, tab, hp, b, D); break;
+    case 64: k_pt_paths<COMPAT, 64, RING><<<grid, 64, 0, st>>>(g, s, tab, hp, b, D, waves); break;
+    case 128: k_pt_paths<COMPAT, 128, RING><<<grid, 128, 0, st>>>(g, s, tab, hp, b, D, waves); break;
     case 512:
-      if constexpr (RING <= 16) k_pt_paths<COMPAT, 512, RING><<<grid, 512, 0, st>>>(g, s, tab, hp, b, D);
+      if constexpr (RING <= 16) k_pt_paths<COMPAT, 512, RING><<<grid, 512, 0, st>>>(g, s, tab, hp, b, D, waves);
       break;
-    default: k_pt_paths<COMPAT, 256, RING><<<grid, 256, 0, st>>>(g, s, tab, hp, b, D); break;
+    default: k_pt_paths<COMPAT, 256, RING><<<grid, 256, 0, st>>>(g, s, tab, hp, b, D, waves); break;
   }
 }
 
@@ -680,17 +693,17 @@ void launch_paths_bs(int grid, int block, hipStream_t st, const TraceGeom& g, co
 // with refill, then shading) or every remaining bounce in one launch (fetch 3
 // at bounce 1, fetch 4 at bounce 2).
 template <bool COMPAT>
-void launch_bounce(bool first, bool count, int fetch, int grid, int block, int ring, hipStream_t st,
+void launch_bounce(int cus, bool first, bool count, int fetch, int grid, int block, int ring, hipStream_t st,
                    const TraceGeom& g, const PtState& s, const CamDev& cam, const HaltonTables& tab,
                    const HaltonParams& hp, int spp, int b, int D, unsigned long long* visits) {
   // the first bounce's camera rays are coherent: a wave's lanes stay in step
   // in the fused kernel, which refilling them one by one would undo
   if (((fetch == 3 && b >= 1) || (fetch == 4 && b >= 2)) && !count && !first) {
-    with_ring(ring, [&](auto R) { launch_paths_bs<COMPAT, decltype(R)::value>(grid, block, st, g, s, tab, hp, b, D); });
+    with_ring(ring, [&](auto R) { launch_paths_bs<COMPAT, decltype(R)::value>(cus, grid, block, st, g, s, tab, hp, b, D); });
     return;
   }
   if ((fetch == 2 || fetch == 4) && !count && !first) {
-    with_ring(ring, [&](auto R) { launch_split_bs<COMPAT, decltype(R)::value>(grid, block, st, g, s, b); });
+    with_ring(ring, [&](auto R) { launch_split_bs<COMPAT, decltype(R)::value>(cus, grid, block, st, g, s, b); });
     const int sgrid = grid * block / kShadeBlock > 0 ? grid * block / kShadeBlock : 1;
     k_pt_shade<COMPAT><<<sgrid, kShadeBlock, 0, st>>>(g, s, tab, hp, b, D);
     return;
@@ -880,10 +893,10 @@ int flg_pathtrace_diffuse(flg_ctx* ctx, const flg_bvh* bvh, const flg_camera* ca
         // the camera-ray bounce apart from the incoherent diffuse bounces
         ScopedTimer tk(timed ? ctx : nullptr, b == 0 ? "pathtrace_first_bounce" : "pathtrace_later_bounces");
         if (compat)
-          launch_bounce<true>(b == 0, count_visits, fmode, pgrid, tb, ring, stream, g, s, cd, tab, hp, cfg->spp,
+          launch_bounce<true>(ctx->num_cus, b == 0, count_visits, fmode, pgrid, tb, ring, stream, g, s, cd, tab, hp, cfg->spp,
                               b, D, visits);
         else
-          launch_bounce<false>(b == 0, count_visits, fmode, pgrid, tb, ring, stream, g, s, cd, tab, hp, cfg->spp,
+          launch_bounce<false>(ctx->num_cus, b == 0, count_visits, fmode, pgrid, tb, ring, stream, g, s, cd, tab, hp, cfg->spp,
                                b, D, visits);
         // that launch ran every remaining bounce
         if (!count_visits && ((fmode == 3 && b >= 1) || (fmode == 4 && b >= 2))) break;
