@@ -354,12 +354,19 @@ __global__ __launch_bounds__(256) void k_svol(VolDev v, LightsDev L, HaltonTable
 //   idle     the path is complete: write it, take the next one.
 // The estimator's loops written as loops inside loops (a whole walk of every
 // lane, then a whole scattering event) kept 25% of the lanes active in a kernel
-// bound by VALU issue, since each loop runs to its longest lane; here the
-// scatter, end and idle phases wait until a share of the wave is due.  Every
-// path makes the draws and operations of svol_begin and svol_step in their
-// order, so the bits are theirs.  256^3 fBm frame, 512 x 512 at 64 spp: 8.55 ms
-// against 13.2 ms (4.4 G wave instructions against 5.3 G, lanes active 0.40
-// against 0.25); 4 or 6 waves per SIMD within 2% of 5.
+// bound by VALU issue, since each loop runs to its longest lane; here a wave
+// runs the phase that most of its lanes are due for.  Every path makes the
+// draws and operations of svol_begin and svol_step in their order, so the bits
+// are theirs.  256^3 fBm frame, 512 x 512 at 64 spp: 6.60 ms against 13.0 ms;
+// 4 or 6 waves per SIMD within 2% of 5.
+//
+// The phase with the most lanes, not one that has a fixed number of them: with
+// the scatter, end and idle phases due at 24 lanes that frame took 6.83 ms, a
+// medium eight times as dense 26.1 ms against 24.1, its 15% sparse 128^3 one 34.9
+// against 32.0, and a constant grid, whose walks are a step each, 4.63 ms against
+// 4.20 (4.39 as loops inside loops; 512 x 512 at 64 spp, depth 8).  The same grid
+// at 256 x 256, 16 spp and depth 4 stays slower than those loops, 396 against 340
+// us: with one-step walks their lanes never part.
 enum : int { kLaneWalk, kLaneScatter, kLaneEnd, kLaneIdle, kLaneOut };
 enum : int { kWalkCamera, kWalkShadow, kWalkDelta, kWalkNone };  // None: a scattering event without a shadow ray
 
@@ -478,14 +485,19 @@ FLG_D void lane_end(const VolDev& v, const LightsDev& L, const HaltonTables& tab
   else lane_walk(v, kWalkDelta, a.s.o, a.s.d, kInf, a);
 }
 
-// Lanes due for a phase before it runs, while others can walk.  256^3 fBm frame
-// and a 200 x 151 film of 90,600 tasks: 24 of each 8.55 and 1.12 ms, 32 and 24
-// for idle 8.46 and 1.24, 40 and 32 8.69 and 1.30 (16 of each, with slower long
-// walks: 7% slower on the first).
-constexpr int kScatterDue = 24, kEndDue = 24, kIdleDue = 24;
+constexpr int kSvolWaves = 5;  // per SIMD
 
-template <bool COUNT, bool FILM>
-__global__ __launch_bounds__(256, 5) void k_svol_regen(VolDev v, LightsDev L, HaltonTables tab_g,
+// Paths a wave claims at once.  While the whole launch has no more than two
+// paths for every lane that the device holds (kSvolWaves waves per SIMD), a wave
+// claims one per lane, so that the paths spread over all waves: the time is that
+// of a wave's chain of phases then.  200 x 200 at 4 spp on the 256^3 fBm grid 685
+// us against 823 with kVolChunk, 128 x 128 at 4 spp on a constant grid 418 against
+// 577 (535 as loops inside loops); 512 x 512 at 64 spp on the fBm grid 7.01
+// against 6.60 ms.
+constexpr uint32_t kSvolSmallChunk = 64;
+
+template <bool COUNT, bool FILM, uint32_t CHUNK>
+__global__ __launch_bounds__(256, kSvolWaves) void k_svol_regen(VolDev v, LightsDev L, HaltonTables tab_g,
                                                     HaltonParams hp, CamDevV cam, int32_t tasks,
                                                     int32_t max_depth, float* lpath, float2* fpos,
                                                     unsigned int* next_path,
@@ -502,9 +514,17 @@ __global__ __launch_bounds__(256, 5) void k_svol_regen(VolDev v, LightsDev L, Ha
   // every trip advances some lane, and the path counter only grows: a wave
   // leaves once its lanes have drawn indices past npaths
   while (true) {
-    const uint64_t mw = __ballot(a.state == kLaneWalk), ms = __ballot(a.state == kLaneScatter),
-                   me = __ballot(a.state == kLaneEnd), mi = __ballot(a.state == kLaneIdle);
-    if (!(mw | ms | me | mi)) break;
+    int phase = kLaneOut, most = 0;
+    auto offer = [&](int state) {
+      const int n = __popcll(__ballot(a.state == state));
+      phase = n > most ? state : phase;
+      most = n > most ? n : most;
+    };
+    offer(kLaneIdle);
+    offer(kLaneEnd);
+    offer(kLaneScatter);
+    offer(kLaneWalk);
+    if (phase == kLaneOut) break;
     uint64_t ml = __ballot(a.state == kLaneWalk && walk_is_long(tab, a.s.ps, a.w));
     if (ml) {
       const V3 o = a.walk == kWalkCamera ? cam.pos : a.s.o;
@@ -517,7 +537,7 @@ __global__ __launch_bounds__(256, 5) void k_svol_regen(VolDev v, LightsDev L, Ha
       }
       continue;
     }
-    if (mi && (__popcll(mi) >= kIdleDue || !(mw | ms | me))) {
+    if (phase == kLaneIdle) {
       // indices for the idle lanes: the rest of the wave's chunk, then a fresh
       // one; a lane that goes on to its task's sample 1 leaves its index unused
       // by keeping it out of the count
@@ -534,13 +554,13 @@ __global__ __launch_bounds__(256, 5) void k_svol_regen(VolDev v, LightsDev L, Ha
         const uint32_t r = (uint32_t)__popcll(mt & ((1ull << lane) - 1ull));
         uint32_t fresh = 0;
         if (rem < nw) {
-          if (lane == 0) fresh = atomicAdd(next_path, kVolChunk);
+          if (lane == 0) fresh = atomicAdd(next_path, CHUNK);
           fresh = __builtin_amdgcn_readfirstlane(fresh);
         }
         const uint32_t mine = r < rem ? cursor + r : fresh + (r - rem);
         if (rem < nw) {
           cursor = fresh + (nw - rem);
-          end = fresh + kVolChunk;
+          end = fresh + CHUNK;
         } else {
           cursor += nw;
         }
@@ -549,9 +569,9 @@ __global__ __launch_bounds__(256, 5) void k_svol_regen(VolDev v, LightsDev L, Ha
           else a.state = kLaneOut;
         }
       }
-    } else if (me && (__popcll(me) >= kEndDue || !(mw | ms))) {
+    } else if (phase == kLaneEnd) {
       if (a.state == kLaneEnd) lane_end(v, L, tab, hp, max_depth, a);
-    } else if (ms && (__popcll(ms) >= kScatterDue || !mw)) {
+    } else if (phase == kLaneScatter) {
       if (a.state == kLaneScatter) lane_scatter(v, L, tab, hp, a);
     } else {
       if (a.state == kLaneWalk) lane_step<COUNT>(v, tab, hp, cam, a, nlook);
@@ -1214,13 +1234,18 @@ static int volpath_render(flg_ctx* ctx, flg_volume* vol, const flg_vol_scene* sc
     ScopedTimer tm(ctx, "volpath_paths");
     const int blocks1 = (int)div_up(npaths, 256);
     const int blocks2 = (int)std::min<int64_t>(div_up(npaths, 256), (int64_t)ctx->num_cus * 8);
+    const bool small = npaths <= (int64_t)2 * 64 * 4 * kSvolWaves * ctx->num_cus;
 #define FLG_SVOL_LAUNCH(C, F)                                                                              \
   if (sched == 1)                                                                                          \
     k_svol<C, F><<<blocks1, 256, 0, ctx->stream>>>(v, L, tab, hp, cam, tasks, cfg->max_depth, lpath, fpos, \
                                                    nl);                                                    \
+  else if (small)                                                                                          \
+    k_svol_regen<C, F, kSvolSmallChunk><<<blocks2, 256, 0, ctx->stream>>>(v, L, tab, hp, cam, tasks,       \
+                                                                          cfg->max_depth, lpath, fpos,     \
+                                                                          next_path, nl);                  \
   else                                                                                                     \
-    k_svol_regen<C, F><<<blocks2, 256, 0, ctx->stream>>>(v, L, tab, hp, cam, tasks, cfg->max_depth, lpath, \
-                                                         fpos, next_path, nl);
+    k_svol_regen<C, F, kVolChunk><<<blocks2, 256, 0, ctx->stream>>>(v, L, tab, hp, cam, tasks,             \
+                                                                    cfg->max_depth, lpath, fpos, next_path, nl);
     if (count && film) {
       FLG_SVOL_LAUNCH(true, true)
     } else if (count) {
