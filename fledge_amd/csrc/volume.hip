@@ -19,37 +19,55 @@ namespace flg {
 namespace {
 
 constexpr int kEnvN = 512;
-// The quads of a dense grid with its zero border, one lane per quad: bound by
-// the 16 bytes it writes (its four reads share lines with its neighbours').
-__global__ __launch_bounds__(256) void k_quads(const float* src, float4* dst, int nx, int ny, int nz) {
-  const int px = nx + 2, qy = ny + 1, qz = nz + 1;
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int64_t tot = (int64_t)px * qy * qz;
-  if (i >= tot) return;
-  const int x = (int)(i % px) - 1, y = (int)((i / px) % qy) - 1, z = (int)(i / ((int64_t)px * qy)) - 1;
-  float v[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int yy = y + (c & 1), zz = z + (c >> 1);
-    const bool in = x >= 0 && x < nx && yy >= 0 && yy < ny && zz >= 0 && zz < nz;
-    v[c] = in ? src[((int64_t)zz * ny + yy) * nx + x] : 0.0f;
-  }
-  dst[i] = make_float4(v[0], v[1], v[2], v[3]);
-}
-
-__global__ __launch_bounds__(256) void k_max(const float* src, int64_t n, float* out) {
+// The quads of a dense grid with its zero border, and the greatest voxel of each
+// block.  A lane makes kQuadColumn quads above one another, so that it reads two
+// voxels a quad instead of four and finds its place, two divisions, once for
+// them; the maximum takes no pass of its own.  Bound by the 16 bytes a quad that
+// it writes.  flg_volume_update of 192^3, 256^3 and 512^3 voxels: 54, 95 and 640
+// us, with a lane per quad and a pass for the maximum 72, 144 and 1167 us (60, 102
+// and 870 us for a padded grid of floats, a quarter of the bytes).  STREAM: past
+// the caches, for grids that the 256 MB of the memory-side cache don't hold (256^3
+// 115 us without; below that size the same, and a frame after it may find the
+// quads there).
+constexpr int kQuadColumn = 8;
+constexpr int64_t kStreamBytes = (int64_t)256 << 20;
+template <bool STREAM>
+__global__ __launch_bounds__(256) void k_quads(const float* src, float4* dst, int nx, int ny, int nz, float* out) {
   __shared__ float red[4];
+  const uint32_t px = (uint32_t)nx + 2u, qy = (uint32_t)ny + 1u, qz = (uint32_t)nz + 1u;
+  const uint32_t n = px * qy * ((qz + kQuadColumn - 1) / kQuadColumn);
   float m = -3.402823466e+38f;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    m = smax(m, src[i]);
+  for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
+    const uint32_t row = t / px, c = row / qy;
+    const int x = (int)(t - row * px) - 1, y = (int)(row - c * qy) - 1, z0 = (int)(c * kQuadColumn) - 1;
+    const bool in0 = x >= 0 && x < nx && y >= 0, in1 = x >= 0 && x < nx && y + 1 < ny;
+    float a[kQuadColumn + 1], b[kQuadColumn + 1];  // the voxels at y and at y + 1, z0 on
+#pragma unroll
+    for (int k = 0; k <= kQuadColumn; ++k) {
+      const int z = z0 + k;
+      const bool in = z >= 0 && z < nz;
+      const float* p = src + ((int64_t)z * ny + y) * nx + x;
+      a[k] = in && in0 ? p[0] : 0.0f;
+      b[k] = in && in1 ? p[nx] : 0.0f;
+    }
+    float4* q = dst + (size_t)c * kQuadColumn * qy * px + (size_t)(y + 1) * px + (uint32_t)(x + 1);
+#pragma unroll
+    for (int k = 0; k < kQuadColumn; ++k) {
+      const int z = z0 + k;
+      if (z < nz) {
+        typedef float F4 __attribute__((ext_vector_type(4)));
+        const F4 v = {a[k], b[k], a[k + 1], b[k + 1]};
+        F4* at = reinterpret_cast<F4*>(q + (size_t)k * qy * px);
+        if (STREAM) __builtin_nontemporal_store(v, at);
+        else *at = v;
+      }
+      if (in0 && z >= 0 && z < nz) m = smax(m, a[k]);
+    }
+  }
   for (int o = 32; o >= 1; o >>= 1) m = smax(m, __shfl_xor(m, o, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float r = smax(smax(red[0], red[1]), smax(red[2], red[3]));
-    out[blockIdx.x] = r;
-  }
+  if (threadIdx.x == 0) out[blockIdx.x] = smax(smax(red[0], red[1]), smax(red[2], red[3]));
 }
 
 // Dist1D ctor (distribution.hpp:14-22)
@@ -1050,16 +1068,23 @@ int make_lights(flg_ctx* ctx, flg_volume* vol, const flg_vol_scene* sc, LightsDe
   return FLG_OK;
 }
 
-int refresh_max(flg_ctx* ctx, flg_volume* vol, const float* d_density) {
+// Makes a dense volume's quads from its voxels and takes their maximum.
+int dense_fill(flg_ctx* ctx, flg_volume* vol, const float* d_density) {
+  const int64_t lanes =
+      (int64_t)(vol->nx + 2) * (vol->ny + 1) * ((vol->nz + 1 + kQuadColumn - 1) / kQuadColumn);
+  const int blocks = (int)std::min<int64_t>(div_up(lanes, 256), (int64_t)ctx->num_cus * 8);
   int st = FLG_OK;
-  const int64_t tot = (int64_t)vol->nx * vol->ny * vol->nz;
-  const int blocks = 512;
-  float* part = (float*)scratch(ctx, "vol_max", blocks * 4, &st);
+  float* part = (float*)scratch(ctx, "vol_max", (size_t)blocks * 4, &st);
   if (!part) return st;
-  k_max<<<blocks, 256, 0, ctx->stream>>>(d_density, tot, part);
+  // rows of a wave's lanes at least: a shorter row's stores fill no lines by themselves
+  const int64_t bytes = (int64_t)(vol->nx + 2) * (vol->ny + 1) * (vol->nz + 1) * (int64_t)sizeof(float4);
+  if (bytes > kStreamBytes && vol->nx >= 64)
+    k_quads<true><<<blocks, 256, 0, ctx->stream>>>(d_density, vol->quads, vol->nx, vol->ny, vol->nz, part);
+  else
+    k_quads<false><<<blocks, 256, 0, ctx->stream>>>(d_density, vol->quads, vol->nx, vol->ny, vol->nz, part);
   FLG_CHECK_LAUNCH(ctx);
   std::vector<float> h(blocks);
-  FLG_CHECK_HIP(ctx, hipMemcpyAsync(h.data(), part, blocks * 4, hipMemcpyDeviceToHost, ctx->stream));
+  FLG_CHECK_HIP(ctx, hipMemcpyAsync(h.data(), part, h.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
   FLG_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
   float m = -3.402823466e+38f;
   for (float x : h) m = smax(m, x);
@@ -1355,10 +1380,7 @@ int flg_volume_update(flg_ctx* ctx, flg_volume* vol, const float* d_density) {
     if (!ctx || !vol || !d_density) return set_error(ctx, FLG_ERR_INVALID, "flg_volume_update: bad arguments");
     if (vol->bmap)
       return set_error(ctx, FLG_ERR_INVALID, "flg_volume_update: a sparse volume takes flg_volume_update_sparse");
-    const int64_t tot = (int64_t)(vol->nx + 2) * (vol->ny + 1) * (vol->nz + 1);
-    k_quads<<<div_up(tot, 256), 256, 0, ctx->stream>>>(d_density, vol->quads, vol->nx, vol->ny, vol->nz);
-    FLG_CHECK_LAUNCH(ctx);
-    return refresh_max(ctx, vol, d_density);
+    return dense_fill(ctx, vol, d_density);
   });
 }
 
