@@ -480,7 +480,7 @@ struct BuildOut {
   float* ctot;         // per chunk: union of its leaves
   int32_t* cross;      // the crossing nodes, in no order
   uint32_t* ncross;    // how many
-  uint32_t* nonfinite; // set if a vertex of a triangle is infinite or NaN
+  uint32_t* nonfinite; // per segment: set if a vertex of a triangle is infinite or NaN
 };
 
 // Child references of a node split at gamma.
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_refit_chunks(const SegDesc* s
     lb[k] = Box{vmin(vmin(va[k], vb[k]), vc[k]), vmax(vmax(va[k], vb[k]), vc[k])};
     const float size = ((fabsf(va[k].x) + fabsf(va[k].y)) + (fabsf(va[k].z) + fabsf(vb[k].x))) +
                        ((fabsf(vb[k].y) + fabsf(vb[k].z)) + (fabsf(vc[k].x) + fabsf(vc[k].y))) + fabsf(vc[k].z);
-    if (!(size < __builtin_inff())) *o.nonfinite = 1u;
+    if (!(size < __builtin_inff())) o.nonfinite[chunk_seg[b]] = 1u;
     if (lslot[k] == kNoParent) continue;
     const uint32_t x = lslot[k] >> 1;
     if (inside(x)) put_box(&sbox[x - A][(lslot[k] & 1) * 6], lb[k]);
@@ -984,7 +984,7 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
   const size_t hist_words = (size_t)nseg * kPasses * kDigits;
   const size_t status_words = (size_t)kPasses * tile_total * kDigits;
   const size_t flag_words = (2 * N + 3) / 4;  // two byte arrays
-  const size_t zero_words = hist_words + status_words + kPasses + 3 + flag_words;
+  const size_t zero_words = hist_words + status_words + kPasses + 2 + nseg + flag_words;
   const size_t so_zero = stake(zero_words * 4);
   char* sc = (char*)scratch(ctx, "lbvh_build", s_off ? s_off : 256, &st);
   if (!sc) return fail(st);
@@ -1005,7 +1005,7 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
   uint32_t* err = counters + kPasses;
   uint32_t* ncross = err + 1;
   uint32_t* nonfinite = ncross + 1;
-  uint8_t* want = (uint8_t*)(nonfinite + 1);
+  uint8_t* want = (uint8_t*)(nonfinite + nseg);
 
   BuildOut o;
   o.nodes = (BNode*)(base + o_nodes);
@@ -1078,12 +1078,12 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
     if (e != hipSuccess) return fail(check_hip(ctx, e, "lbvh build kernels"));
   }
   std::vector<float> hgb((size_t)nseg * 6, 0.0f);
-  uint32_t herr[3] = {0, 0, 0};  // err, ncross, nonfinite
+  std::vector<uint32_t> words(2 + (size_t)nseg, 0u);  // err, ncross, nonfinite
   if (hipMemcpyAsync(hgb.data(), gb, hgb.size() * 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-      hipMemcpyAsync(herr, err, sizeof herr, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+      hipMemcpyAsync(words.data(), err, words.size() * 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
       hipStreamSynchronize(ctx->stream) != hipSuccess)
     return fail(set_error(ctx, FLG_ERR_HIP, "lbvh build: synchronisation failed"));
-  if (herr[0]) return fail(set_error(ctx, FLG_ERR_HIP, "lbvh build: a sort tile's look-back did not complete"));
+  if (words[0]) return fail(set_error(ctx, FLG_ERR_HIP, "lbvh build: a sort tile's look-back did not complete"));
 
   SharedBlock* sb = new SharedBlock;
   sb->ptr = blockp;
@@ -1097,9 +1097,9 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
     h->flags = flags;
     for (int k = 0; k < 6; ++k) h->bound[k] = d.ntris > 0 ? hgb[6 * s + k] : 0.0f;
     h->nodes = o.nodes + d.node_base;
-    // coordinates beyond the range of the wide nodes' grids and margins, or a
-    // mesh of the batch with infinite or NaN ones: binary nodes only
-    bool ranged = !herr[2];
+    // coordinates beyond the range of the wide nodes' grids and margins, or
+    // infinite or NaN ones: binary nodes only
+    bool ranged = !words[2 + s];
     for (int k = 0; k < 6; ++k) ranged = ranged && std::fabs(h->bound[k]) <= 0x1p40f;
     h->wide = o.wide && ranged ? o.wide + d.node_base : nullptr;
     h->tris = o.tris + d.tri_base;

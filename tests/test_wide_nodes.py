@@ -76,3 +76,26 @@ def test_wide_nodes_gpu(ctx, mesh):
         oid, ot = o.trace(rays[:n])
         assert np.array_equal(gid, oid)
         assert np.array_equal(gt.view(np.uint32), ot.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_unbounded_vertices(ctx, value):
+    """Meshes with a vertex that is not finite, alone and in a batch with finite
+    ones (each mesh of a batch picks its nodes for itself): ids and t bit-equal to
+    the oracle's binary traversal."""
+    print("unbounded vertices %r" % value, flush=True)
+    sizes, bad = (1500, 700, 2049, 1), (1, 2)
+    meshes = [api.gen_soup(n, initseq=60 + k) for k, n in enumerate(sizes)]
+    for k in bad:
+        meshes[k][0][9 * (sizes[k] // 2) + 4] = value
+    up = [(torch.from_numpy(v).cuda(), torch.from_numpy(i).cuda()) for v, i in meshes]
+    rays = _rays(meshes[0][0], 8000, 5)
+    for k, b in enumerate(api.LBVH.build_batched(ctx, up)):
+        alone = api.LBVH.build(ctx, *up[k])
+        oid, ot = orc.Lbvh(*meshes[k]).trace(rays)
+        for g in (b, alone):
+            gid, gt = api.hits_as_numpy(g.trace(torch.from_numpy(rays).cuda()))
+            assert np.array_equal(gid, oid)
+            assert np.array_equal(gt.view(np.uint32), ot.view(np.uint32))
+        assert sizes[k] == 1 or (oid >= 0).any()  # the small triangle lies off every ray
