@@ -1114,7 +1114,7 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
     h->leaf_parent = o.leaf_parent + d.tri_base;
     h->gbound = gb + 6 * s;
     h->bytes = (uint64_t)d.ntris * (sizeof(BTri) + 5 * 4) +
-               (uint64_t)(d.ntris > 0 ? d.ntris - 1 : 0) * (sizeof(BNode) + 17);
+               (uint64_t)(d.ntris > 0 ? d.ntris - 1 : 0) * (sizeof(BNode) + 17 + (o.wide ? sizeof(WNode) : 0));
     h->block = sb;
     out[s] = h;
   }

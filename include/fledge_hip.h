@@ -137,7 +137,7 @@ FLG_API int flg_lbvh_build_batched(flg_ctx* ctx, const flg_mesh_desc* h_meshes, 
 typedef struct flg_lbvh_info {
   int32_t ntris;
   float bound[6]; /* global bound lo.xyz, hi.xyz */
-  uint64_t device_bytes;
+  uint64_t device_bytes; /* of the BVH's arrays: 213 per triangle, 149 without wide nodes */
 } flg_lbvh_info;
 FLG_API int flg_lbvh_get_info(flg_bvh* bvh, flg_lbvh_info* out);
 

@@ -99,3 +99,14 @@ def test_unbounded_vertices(ctx, value):
             assert np.array_equal(gid, oid)
             assert np.array_equal(gt.view(np.uint32), ot.view(np.uint32))
         assert sizes[k] == 1 or (oid >= 0).any()  # the small triangle lies off every ray
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 1500])
+def test_device_bytes(ctx, n):
+    """flg_lbvh_info.device_bytes counts every array of the build: 48 bytes of
+    triangle and 20 of leaf arrays a triangle; 64 of binary node, 64 of wide node
+    and 17 of node arrays a node."""
+    v, i = api.gen_soup(n)
+    b = api.LBVH.build(ctx, torch.from_numpy(v).cuda(), torch.from_numpy(i).cuda())
+    assert b.info().device_bytes == 68 * n + 145 * (n - 1)
