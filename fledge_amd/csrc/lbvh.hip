@@ -979,7 +979,6 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
   const size_t so_k0 = stake(N * 4), so_v0 = stake(N * 4), so_k1 = stake(N * 4), so_v1 = stake(N * 4);
   const size_t so_ninfo = stake(NI * 4), so_lslot = stake(N * 4);
   const size_t so_pre = stake(N * 24), so_suf = stake(N * 24), so_ctot = stake(chunk_total * 24);
-  const size_t so_cross = stake(NI * 4);
   const size_t so_blkseg = stake(blk_total * 4), so_chunkseg = stake(chunk_total * 4);
   const size_t hist_words = (size_t)nseg * kPasses * kDigits;
   const size_t status_words = (size_t)kPasses * tile_total * kDigits;
@@ -1027,7 +1026,7 @@ static int build_segments(flg_ctx* ctx, const flg_mesh_desc* meshes, int nseg, u
   o.pre = (float*)(sc + so_pre);
   o.suf = (float*)(sc + so_suf);
   o.ctot = (float*)(sc + so_ctot);
-  o.cross = (int32_t*)(sc + so_cross);
+  o.cross = (int32_t*)k1;  // the sort is done with it
   o.ncross = ncross;
   o.nonfinite = nonfinite;
   float* gb = (float*)(base + o_gb);
