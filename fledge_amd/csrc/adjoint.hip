@@ -166,10 +166,10 @@ FLG_D void diff_finish(const DiffDev& D, uint32_t p, const DiffPath& s, float* l
 
 // One lane per path sample.
 template <bool ADJ>
-__global__ __launch_bounds__(256) void k_diff(DiffDev D, LightsDev L, HaltonTables tab_g,
-                                              HaltonParams hp, CamDevV cam, int32_t spp,
-                                              int32_t max_depth, float* lpath,
-                                              const float* dl_drgb, float* grad, float* galpha) {
+__global__ __launch_bounds__(kDiffBlock) void k_diff(DiffDev D, LightsDev L, HaltonTables tab_g,
+                                                     HaltonParams hp, CamDevV cam, int32_t spp,
+                                                     int32_t max_depth, float* lpath,
+                                                     const float* dl_drgb, float* grad, float* galpha) {
   __shared__ int2 lds_primes[kLocalPrimes];
   const HaltonTables tab = stage_halton(tab_g, lds_primes);
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -186,11 +186,11 @@ __global__ __launch_bounds__(256) void k_diff(DiffDev D, LightsDev L, HaltonTabl
 
 // Persistent lanes with path regeneration (regen_loop); same per-path code.
 template <bool ADJ>
-__global__ __launch_bounds__(256) void k_diff_regen(DiffDev D, LightsDev L, HaltonTables tab_g,
-                                                    HaltonParams hp, CamDevV cam, int32_t spp,
-                                                    int32_t max_depth, float* lpath,
-                                                    const float* dl_drgb, float* grad, float* galpha,
-                                                    unsigned int* next_path) {
+__global__ __launch_bounds__(kDiffBlock) void k_diff_regen(DiffDev D, LightsDev L, HaltonTables tab_g,
+                                                           HaltonParams hp, CamDevV cam, int32_t spp,
+                                                           int32_t max_depth, float* lpath,
+                                                           const float* dl_drgb, float* grad, float* galpha,
+                                                           unsigned int* next_path) {
   __shared__ int2 lds_primes[kLocalPrimes];
   const HaltonTables tab = stage_halton(tab_g, lds_primes);
   const uint32_t npaths = (uint32_t)((int64_t)cam.w * cam.h * spp);
@@ -217,17 +217,17 @@ int launch_diff(flg_ctx* ctx, const flg_render_cfg* cfg, const DiffDev& D, const
   const int64_t npaths = (int64_t)cfg->width * cfg->height * cfg->spp;
   const int sched = cfg->schedule ? cfg->schedule : 2;
   if (sched == 1) {
-    k_diff<ADJ><<<div_up(npaths, 256), 256, 0, ctx->stream>>>(D, L, tab, hp, cam, cfg->spp, cfg->max_depth,
-                                                               lpath, dl, grad, galpha);
+    k_diff<ADJ><<<div_up(npaths, kDiffBlock), kDiffBlock, 0, ctx->stream>>>(D, L, tab, hp, cam, cfg->spp,
+                                                                            cfg->max_depth, lpath, dl, grad, galpha);
     return FLG_OK;
   }
   int st = FLG_OK;
   unsigned int* counter = (unsigned int*)scratch(ctx, ADJ ? "diff_counter_adj" : "diff_counter_fwd", 256, &st);
   if (!counter) return st;
   k_zero_counter<<<1, 1, 0, ctx->stream>>>(counter);
-  const int grid = (int)std::min<int64_t>(div_up(npaths, 256), (int64_t)ctx->num_cus * 8);
-  k_diff_regen<ADJ><<<grid, 256, 0, ctx->stream>>>(D, L, tab, hp, cam, cfg->spp, cfg->max_depth, lpath, dl,
-                                                   grad, galpha, counter);
+  const int grid = (int)std::min<int64_t>(div_up(npaths, kDiffBlock), (int64_t)ctx->num_cus * 8);
+  k_diff_regen<ADJ><<<grid, kDiffBlock, 0, ctx->stream>>>(D, L, tab, hp, cam, cfg->spp, cfg->max_depth, lpath, dl,
+                                                          grad, galpha, counter);
   return FLG_OK;
 }
 

@@ -79,7 +79,7 @@ FLG_D int64_t grad_at(const DiffDev& D, int x, int y, int z) {
   return ((int64_t)slot << (3 * sh)) + (((z & m) << (2 * sh)) | ((y & m) << sh) | (x & m));
 }
 
-constexpr int kDiffBlock = 256;  // most threads of a block that deposits
+constexpr int kDiffBlock = 256;  // most threads of a block that deposits (its LDS rows)
 constexpr int kDepositShare = 32;  // lookups handed over at a time in a wave
 
 // Gradient scatter: g * trilinear weight for the eight corners of the lookup.

@@ -768,6 +768,8 @@ FLG_D void vpd_finish(const DiffDev& D, uint32_t p, const DiffVPath& s, float* l
   }
 }
 
+static_assert(kMeshBlock <= kDiffBlock, "deposit has LDS rows for the waves of kDiffBlock threads");
+
 // One lane per path sample.
 template <bool ADJ, bool COMPAT>
 __global__ __launch_bounds__(kMeshBlock, kMeshWaves) void k_vpdiff(TraceGeom g, DiffDev D, LightsDev L, HaltonTables tab_g,
