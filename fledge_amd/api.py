@@ -124,22 +124,10 @@ class LBVH:
             raise ValueError("ind%s: indices into an empty vertex array" % k)
 
     @staticmethod
-    def _check_indices(meshes):
-        """Every index in [0, nverts): one reduction per mesh, then one sync."""
-        bad = []
-        for k, (v, ind) in enumerate(meshes):
-            if ind.numel():
-                lo, hi = torch.aminmax(ind)
-                bad.append((k, lo, hi, v.numel() // 3))
-        for k, lo, hi, nv in bad:
-            if int(lo) < 0 or int(hi) >= nv:
-                raise ValueError("mesh %d: vertex indices in [%d, %d] outside [0, %d)" % (k, int(lo), int(hi), nv))
-
-    @staticmethod
     def _check_ranges(ctx, descs, n):
-        """_check_indices for n mesh descriptors of `ctx`'s device: one launch
-        and one synchronisation for all of them, after the current stream's
-        work where that is not the context's."""
+        """Every index of n meshes in [0, nverts): one launch and one
+        synchronisation for all of them, after the current stream's work where
+        that is not the context's."""
         current = torch.cuda.current_stream(ctx.device)
         if current.cuda_stream != (ctx.stream or 0):
             current.synchronize()

@@ -2,6 +2,7 @@
 wrong dtype, strided views, short outputs, wrong shapes and tensors off the
 context's GPU.  Every check runs before the C ABI is called, so these run on
 the CPU with a context stand-in whose library is never reached."""
+import ctypes
 import types
 
 import pytest
@@ -76,11 +77,32 @@ def test_build_refuses_bad_meshes():
     _raises(lambda: api.LBVH.build_batched(ctx, [(v, i), (v, i.double())]), r"ind\[1\]: dtype")
 
 
-def test_index_range_check():
+def test_index_range_check(monkeypatch):
+    """Both builds check their indices before the native build is reached.  The
+    library is a stand-in on CPU tensors: its ranges are the indices' own."""
+    built = []
+
+    def ranges(h, descs, n, lo, hi):
+        for k in range(n):
+            ind = (ctypes.c_int32 * (3 * descs[k].ntris)).from_address(descs[k].d_ind)
+            lo[k], hi[k] = min(ind), max(ind)
+
+    lib = types.SimpleNamespace(flg_mesh_index_ranges=ranges, flg_lbvh_build=lambda *a: built.append(1),
+                                flg_lbvh_build_batched=lambda *a: built.append(a[2]))
+    ctx = types.SimpleNamespace(device=0, lib=lib, h=None, stream=0, check=lambda st: None)
+    monkeypatch.setattr(api, "check_device", lambda device, **bufs: None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=0))
     v = torch.zeros(9, dtype=torch.float32)
-    api.LBVH._check_indices([(v, torch.tensor([0, 1, 2], dtype=torch.int32))])
-    _raises(lambda: api.LBVH._check_indices([(v, torch.tensor([0, 1, 3], dtype=torch.int32))]), "outside")
-    _raises(lambda: api.LBVH._check_indices([(v, torch.tensor([-1, 1, 2], dtype=torch.int32))]), "outside")
+    good, high, low = (torch.tensor(t, dtype=torch.int32) for t in ([0, 1, 2], [0, 1, 3], [-1, 1, 2]))
+    api.LBVH.build(ctx, v, good)
+    api.LBVH.build_batched(ctx, [(v, good), (v, good)])
+    assert built == [1, 2]
+    for bad in (high, low):
+        _raises(lambda: api.LBVH.build(ctx, v, bad), "mesh 0: .* outside")
+        _raises(lambda: api.LBVH.build_batched(ctx, [(v, good), (v, bad)]), "mesh 1: .* outside")
+    assert built == [1, 2]
+    api.LBVH.build(ctx, v, high, check_indices=False)
+    assert built == [1, 2, 1]
 
 
 def test_scene_camera_and_volume_wrappers_refuse_bad_buffers():
