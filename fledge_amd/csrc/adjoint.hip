@@ -362,12 +362,13 @@ int diff_prepare(flg_ctx* ctx, flg_volume* vol, const flg_volume* proposal, cons
   return FLG_OK;
 }
 
-// When cells pay.  Clearing and gathering them costs about 10 ps a cell, and a
-// path's deposits save about 2 ns: forward and adjoint of 128^3 at 32.8 cells a
-// path 2.56 ms with cells and 2.52 without, of 256^3 at 32.4 cells 3.5 and 4.2
-// ms, at 64.8 cells 3.4 and 3.2 ms.  At most 2 GB.  Not under capture: a graph
-// would keep the cells' address past a later, larger call, which replaces them;
-// it keeps to the caller's buffers.
+// When cells pay: while there are few of them for the paths that deposit.
+// Forward and adjoint with cells and without, 128^3 at 32.8 cells a path: 2.56
+// and 2.52 ms; 256^3 at 32.4 cells a path 3.5 and 4.2 ms, at 64.8 cells 3.4 and
+// 3.2 ms; 128^3 at 2 cells a path 3.4 and 5.8 ms.  So the line is at 32, where the
+// smaller grid is even.  At most 2 GB.  Not under capture: a graph would keep the
+// cells' address past a later, larger call, which replaces them; it keeps to the
+// caller's buffers.
 constexpr int64_t kMaxCells = (int64_t)1 << 26;
 constexpr int64_t kCellsPerPath = 32;
 

@@ -107,8 +107,10 @@ FLG_HD V3 stable_triangle_normal(V3 a, V3 b, V3 c) {
 
 // On the device the three quotients float(x / sqrt(sq)) come from one
 // reciprocal square root, refined to y = (1 + e) / sqrt(sq) with |e| below
-// 2^-51: one third-order step on the hardware's approximation (2^-14 would
-// do).  x y then differs from the correctly rounded x / sqrt(sq) by fewer
+// 2^-51 by one third-order step on the hardware's approximation.  The step
+// leaves 2.5 d^3 of a relative error d, and its own rounding: that asks for d
+// below 2^-17.5, and the instruction's is below 2^-24.1 (2^27 inputs over 256
+// binades).  x y then differs from the correctly rounded x / sqrt(sq) by fewer
 // than 8 units in the last place of a double, so it rounds to the same float
 // unless its low 29 bits lie within 8 of the halfway point between two
 // floats; those, results below the normal floats (where the halfway points lie
