@@ -8,7 +8,9 @@ frame; the BVH build and scene generation are outside the timed region.
 
 The metric's other legs are reported under `legs`, each with its own value,
 roofline (algorithmic bytes over the kernel's HIP-event time, against the
-8 TB/s HBM peak) and CPU baseline (the CPU restatement of the reference's
+8 TB/s HBM peak; for traversals, whose nodes are not the reference's, the HBM
+bytes of the committed counters where there are any, and the reference's node
+visits as work done) and CPU baseline (the CPU restatement of the reference's
 algorithm timed on this host's cores over a bounded sample):
   vol_path       volumetric path samples/s (256^3 fBm grid, 512^2, 64 spp, depth 32)
   fwd_adjoint    differentiable forward + path-replay adjoint, ms per iteration
@@ -60,6 +62,18 @@ def roofline(achieved_gbs, kernel, bytes_per_unit, unit_name, **extra):
     r = {"bound": "hbm", "achieved": round(achieved_gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
          "frac": round(achieved_gbs / HBM_PEAK_GBS, 5), "traffic": None, "kernel": kernel,
          "algorithmic_bytes_per_" + unit_name: bytes_per_unit}
+    r.update(extra)
+    return r
+
+
+def traversal(reference_gbs, kernel, bytes_per_unit, unit_name, **extra):
+    """The record of a traversal: bound by VALU issue with part of the lanes
+    active.  The reference's visits (64 B a binary node, 36 a triangle test, 40 a
+    ray) per second are work done, not bytes moved: the kernels read one 64-byte
+    node for two levels of them."""
+    r = {"bound": "valu issue", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None, "traffic": None,
+         "kernel": kernel, "reference_bytes_per_" + unit_name: bytes_per_unit,
+         "reference_GBps": round(reference_gbs, 2)}
     r.update(extra)
     return r
 
@@ -199,8 +213,8 @@ def main():
     ctx.profiling(False)
     value = segments / dt / 1e6
 
-    # algorithmic bytes per ray segment: 32 (ray) + 8 (hit) + 64 per node
-    # visit + 36 per triangle test, visits counted by the instrumented kernel
+    # the reference's work per ray segment: 32 (ray) + 8 (hit) + 64 per binary
+    # node visit + 36 per triangle test, counted by the instrumented kernel
     cnt = bvh.pathtrace(cam2, W, H, SPP, DEPTH, count_visits=True, **shape)
     vn = cnt["node_visits"] / segments
     vt = cnt["tri_tests"] / segments
@@ -208,33 +222,25 @@ def main():
     launches_per_frame = trace_launches / args.steps
     avg_launch_ms = trace_ms / trace_launches
     bytes_per_launch = bytes_per_ray * segments / launches_per_frame
-    achieved = bytes_per_launch / (avg_launch_ms * 1e-3) / 1e9
     traffic = measured_traffic()
-    head_roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
-                 "kernel": {1: "k_pt_bounce (closest-hit traversal + diffuse bounce, one launch per bounce)",
-                            2: "k_pt_bounce (first bounce) then k_pt_trace + k_pt_shade per bounce "
-                               "(closest-hit traversal with per-wave ray refill, then the diffuse bounce); "
-                               "a launch = one bounce",
-                            3: "k_pt_bounce (first bounce) then k_pt_paths (every later bounce in one launch: "
-                               "each lane follows its path to the end, refilling from the queue); a launch = "
-                               "one of these two",
-                            4: "k_pt_bounce (first bounce), k_pt_trace + k_pt_shade (second), then k_pt_paths "
-                               "(every later bounce in one launch, each lane following its path to the end); a "
-                               "launch = one of these three"}[(tuning or {}).get("ray_fetch", 4) or 4],
-                 "algorithmic_bytes_per_ray": round(bytes_per_ray, 2),
-                 "node_visits_per_ray": round(vn, 3), "tri_tests_per_ray": round(vt, 3),
-                 "avg_launch_ms": round(avg_launch_ms, 4), "launches_per_frame": launches_per_frame,
-                 "trace_kernel_share": round(trace_ms / max(total_ms, 1e-9), 4),
-                 "launch_shape": tuning, "graph": bool(args.graph)}
+    kernels = {1: "k_pt_bounce (closest-hit traversal + diffuse bounce, one launch per bounce)",
+               2: "k_pt_bounce (first bounce) then k_pt_trace + k_pt_shade per bounce "
+                  "(closest-hit traversal with per-wave ray refill, then the diffuse bounce); "
+                  "a launch = one bounce",
+               3: "k_pt_bounce (first bounce) then k_pt_paths (every later bounce in one launch: "
+                  "each lane follows its path to the end, refilling from the queue); a launch = "
+                  "one of these two",
+               4: "k_pt_bounce (first bounce), k_pt_trace + k_pt_shade (second), then k_pt_paths "
+                  "(every later bounce in one launch, each lane following its path to the end); a "
+                  "launch = one of these three"}[(tuning or {}).get("ray_fetch", 4) or 4]
+    head_roof = traversal(bytes_per_launch / (avg_launch_ms * 1e-3) / 1e9, kernels, round(bytes_per_ray, 2), "ray",
+                          node_visits_per_ray=round(vn, 3), tri_tests_per_ray=round(vt, 3),
+                          avg_launch_ms=round(avg_launch_ms, 4), launches_per_frame=launches_per_frame,
+                          trace_kernel_share=round(trace_ms / max(total_ms, 1e-9), 4), launch_shape=tuning,
+                          graph=bool(args.graph))
     if traffic:
-        # the nodes and triangles stay in the 256 MB MALL and the L2s: HBM
-        # itself moves far fewer bytes than the traversal reads, and the
-        # kernels are limited by VALU issue and lane divergence, not bandwidth
         meas = traffic / (avg_launch_ms * 1e-3) / 1e9
-        head_roof.update({"hbm_measured_GBps": round(meas, 2), "hbm_measured_frac": round(meas / HBM_PEAK_GBS, 5),
-                          "limiter": "VALU issue and lane divergence (per-lane traversal); the algorithmic "
-                                     "bytes are served mostly from L2 and MALL"})
+        head_roof.update({"traffic": traffic, "achieved": round(meas, 2), "frac": round(meas / HBM_PEAK_GBS, 5)})
     incoherent = segments - paths  # every segment after a path's camera ray
     secondary = {
         "first_bounce_ms": round(first_ms / args.steps, 4),
@@ -488,8 +494,8 @@ def bench_primary(ctx, N, api, torch, dev, sync, cpu_jobs, secondary):
     out = {"metric": "closest-hit Mrays/s, 1024^2 jittered primary rays on the 65,536-triangle soup",
            "value": round(R / t / 1e6, 2), "unit": "Mrays/s", "higher_is_better": True,
            "kernel_ms": round(kms, 4),
-           "roofline": roofline(bpr * R / (kms * 1e-3) / 1e9, "k_trace", round(bpr, 2), "ray",
-                                node_visits_per_ray=round(vn, 3), tri_tests_per_ray=round(vt, 3)),
+           "roofline": traversal(bpr * R / (kms * 1e-3) / 1e9, "k_trace", round(bpr, 2), "ray",
+                                 node_visits_per_ray=round(vn, 3), tri_tests_per_ray=round(vt, 3)),
            "cpu_baseline": None}
     rays_h = rays0.cpu().numpy()
 
@@ -544,7 +550,7 @@ def bench_vol(ctx, N, api, torch, dev, sync, cpu_jobs):
            "ms_per_frame": round(t1 * 1e3, 3), "ms_per_frame_lane_per_path": round(t1b * 1e3, 3),
            "ms_per_frame_wavefront_graph": round(t1c * 1e3, 3),
            "kernel_ms": round(kms, 4), "lookups_per_path": round(L, 4),
-           "roofline": roofline(lb / (kms * 1e-3) / 1e9, "k_svol_regen (persistent lanes with path regeneration)",
+           "roofline": roofline(lb / (kms * 1e-3) / 1e9, "k_svol_regen (persistent lanes, a phase at a time)",
                                 round(32 * L + 12 / S1, 3), "path"),
            "cpu_baseline": None}
 
@@ -672,9 +678,9 @@ def bench_combined(ctx, N, api, torch, np, dev, sync, cam2, W, H, profile=False,
     P = W * H * SPPc
     rays = stc["rays"]
     look = stc["lookups"]
-    # algorithmic bytes: per trilinear lookup 32 B of voxels + the 4-byte
+    # the reference's work: per trilinear lookup 32 B of voxels + the 4-byte
     # slot-map entry; per ray traced on the mesh 32 B in + 8 B out, 64 B per
-    # node visit and 36 B per triangle test (counted by the same kernel's
+    # binary node visit and 36 B per triangle test (counted by the same kernel's
     # counting build); 12 B per pixel written
     lb = 36 * look + 40 * rays + 64 * stc["node_visits"] + 36 * stc["tri_tests"] + 12 * W * H
     pool_bytes = origins.shape[0] * 4000 + 65 * 65 * 65 * 32
@@ -686,14 +692,14 @@ def bench_combined(ctx, N, api, torch, np, dev, sync, cam2, W, H, profile=False,
            "lookups_per_path": round(look / P, 3),
            "dense_grid_ms_per_frame": round(td * 1e3, 2), "dense_and_sparse_images_bit_equal": same,
            "active_bricks": int(origins.shape[0]), "grid_bytes_sparse": pool_bytes,
-           "grid_bytes_dense": 514 ** 3 * 4,
+           "grid_bytes_dense": 514 * 513 * 513 * 16,
            "diff_forward_ms": round(tf * 1e3, 2), "adjoint_ms": round(ta * 1e3, 2),
            "fwd_adjoint_over_forward": round((tf + ta) / tc, 3),
-           "roofline": roofline(lb / (kms * 1e-3) / 1e9,
-                                "k_volpath_regen (persistent lanes over the interface mesh and the brick pool)",
-                                round(lb / P, 3), "path",
-                                node_visits_per_ray=round(stc["node_visits"] / rays, 3),
-                                tri_tests_per_ray=round(stc["tri_tests"] / rays, 3)),
+           "roofline": traversal(lb / (kms * 1e-3) / 1e9,
+                                 "k_volpath_regen (persistent lanes over the interface mesh and the brick pool)",
+                                 round(lb / P, 3), "path",
+                                 node_visits_per_ray=round(stc["node_visits"] / rays, 3),
+                                 tri_tests_per_ray=round(stc["tri_tests"] / rays, 3)),
            "cpu_baseline": None}
     bc.close()
     if host_grid is not None:
