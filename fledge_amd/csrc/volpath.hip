@@ -40,6 +40,10 @@ constexpr int kMeshRing = 8;
 // it spill to scratch) measured faster than the 3-4 waves of the unconstrained
 // allocation, and than 5 or 7.
 constexpr int kMeshWaves = 6;
+// The counting build of the phased kernel holds its counters as well: at 6 waves
+// it spilled them, 40.2 ms against 28.3 at 4 on an interface-mesh frame of 2M
+// triangles, 1000 x 1000 at 8 spp (3 waves 34.0, 5 waves 30.3 ms).
+constexpr int kMeshCountWaves = 4;
 
 struct MeshGeom {
   TraceGeom g;
@@ -480,12 +484,9 @@ FLG_D void vp_lane_post(const VolDev& v, const LightsDev& L, const HaltonTables&
 constexpr int kVpDue = 7, kVpBatch = 48;
 
 template <bool COMPAT, bool COUNT, bool FILM>
-__global__ __launch_bounds__(kMeshBlock, kMeshWaves) void k_volpath_regen(TraceGeom g, VolDev v, LightsDev L,
-                                                                        HaltonTables tab_g, HaltonParams hp,
-                                                                        CamDevV cam, int32_t tasks, int32_t max_depth,
-                                                                        float* lpath, float2* fpos,
-                                                                        unsigned int* next_path,
-                                                                        unsigned long long* nlookups) {
+__global__ __launch_bounds__(kMeshBlock, COUNT ? kMeshCountWaves : kMeshWaves) void k_volpath_regen(
+    TraceGeom g, VolDev v, LightsDev L, HaltonTables tab_g, HaltonParams hp, CamDevV cam, int32_t tasks,
+    int32_t max_depth, float* lpath, float2* fpos, unsigned int* next_path, unsigned long long* nlookups) {
   __shared__ int2 lds_primes[kLocalPrimes];
   __shared__ uint2 ring[kMeshBlock * kMeshRing];
   const HaltonTables tab = stage_halton(tab_g, lds_primes);
