@@ -33,16 +33,19 @@ def test_hand_out(ctx, w, h, spp, block, per_cu, fetch):
     assert torch.equal(got["seg_t"].view(torch.int32), want["seg_t"].view(torch.int32))
 
 
-def test_blocks_beyond_the_device_cost_nothing(ctx):
+@pytest.mark.parametrize("count", [False, True])
+def test_blocks_beyond_the_device_cost_nothing(ctx, count):
     """64 blocks of 256 threads a CU against 8, most of which find no ray: 3.6
-    times the frame's time when each of their waves asked one counter."""
+    times the frame's time when each of their waves asked one counter, and twice
+    and more when each added to the visits of a counting frame."""
     bvh = sphere(ctx, 4)
     cam = N.Camera.make((0.0, 0.0, -3.0), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 45.0)
 
     def frame(per_cu):
         torch.cuda.synchronize()
         t = time.perf_counter()
-        bvh.pathtrace(cam, 1280, 720, 4, 8, ray_fetch=2, trace_block=256, blocks_per_cu=per_cu)
+        bvh.pathtrace(cam, 1280, 720, 4, 8, ray_fetch=2, trace_block=256, blocks_per_cu=per_cu,
+                      count_visits=count)
         torch.cuda.synchronize()
         return time.perf_counter() - t
 
