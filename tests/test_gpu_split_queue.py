@@ -27,7 +27,8 @@ def test_hand_out(ctx, w, h, spp, block, per_cu, fetch):
     bvh = sphere(ctx, 4)
     cam = N.Camera.make((0.0, 0.0, -1.6), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 45.0)
     want = bvh.pathtrace(cam, w, h, spp, 3, record=True, ray_fetch=1)
-    got = bvh.pathtrace(cam, w, h, spp, 3, record=True, ray_fetch=fetch, trace_block=block, blocks_per_cu=per_cu)
+    got = bvh.pathtrace(cam, w, h, spp, 3, record=True, ray_fetch=fetch, trace_block=block, blocks_per_cu=per_cu,
+                        stack_mode=2, ring_depth=8)
     assert got["segments"] == want["segments"] > w * h * spp
     assert torch.equal(got["nseg"], want["nseg"]) and torch.equal(got["seg_id"], want["seg_id"])
     assert torch.equal(got["seg_t"].view(torch.int32), want["seg_t"].view(torch.int32))
@@ -44,8 +45,8 @@ def test_blocks_beyond_the_device_cost_nothing(ctx, count):
     def frame(per_cu):
         torch.cuda.synchronize()
         t = time.perf_counter()
-        bvh.pathtrace(cam, 1280, 720, 4, 8, ray_fetch=2, trace_block=256, blocks_per_cu=per_cu,
-                      count_visits=count)
+        bvh.pathtrace(cam, 1280, 720, 4, 8, ray_fetch=2, trace_block=256, blocks_per_cu=per_cu, stack_mode=2,
+                      ring_depth=8, count_visits=count)
         torch.cuda.synchronize()
         return time.perf_counter() - t
 
