@@ -38,7 +38,7 @@ namespace flg {
 // dependent) run at 48 G/s against 14 G/s from the plain grid (z pairs, twice
 // the bytes: 27 G/s; all eight voxels of a cell together, eight times the
 // bytes: 54 G/s), bound by the cache lines they ask the L2s and the MALL for.
-// The 256^3 fBm frame takes 6.96 ms against 8.55 ms.  A brick pool keeps plain
+// The 256^3 fBm frame took 6.83 ms against 8.55 ms.  A brick pool keeps plain
 // floats: its lookups stay within a slot of 4 KB, and as quads the pool took
 // more cache than the shorter loads gave (interface-mesh frame 50.0 against
 // 48.5 ms, a small sparse film 1.21 against 1.12 ms).
@@ -424,8 +424,12 @@ FLG_D V3 lane_of(V3 x, int l) { return v3(lane_of(x.x, l), lane_of(x.y, l), lane
 // The first Halton indices have high dimensions of index / prime: their walks
 // take thousands of minute steps, each a chain of a draw, a logarithm and a
 // lookup of about 1.5 us, and a few such paths set the time of a small frame:
-// with them walked by their lane alone, the 256^3 frame of k_svol_regen took
-// 14.4 instead of 8.55 ms and the film of 90,600 tasks 11.2 instead of 1.12 ms.
+// with them walked by their lane alone, the 256^3 frame of k_svol_regen takes
+// 12.5 instead of 6.5 ms and a film of 90,600 tasks 6.6 instead of 0.66 ms.  Every
+// walk counts for itself, however many lanes of the wave have long ones: with
+// sigma_t from 2 to 512, in dense and in mostly empty grids, frames of 8,192 to
+// 2.1 M paths took 0.09 to 0.59 of their time with every walk by its lane in the
+// estimator's nested loops.
 template <bool COUNT>
 FLG_D WalkEvent walk_wave(const VolDev& v, const HaltonTables& tab, const HaltonParams& hp, int l, PathSampler& ps,
                           V3 o_, V3 d_, bool delta_, Walk& wk, V3* pos_out, uint32_t& nlook) {
